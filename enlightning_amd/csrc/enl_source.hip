@@ -294,7 +294,10 @@ int enl_batch_sample_mics(void* handle, int nmics, const double* mic_x, const do
       const PatchDev& pd = b->hp[p];
       if (pd.level != lev) continue;
       const double lo0 = pd.xlo, lo1 = pd.ylo;
-      const double hi0 = (double)(pd.bi0 + pd.nx) * pd.dx, hi1 = (double)(pd.bj0 + pd.ny) * pd.dy;
+      // the upper bounds from the origin of the index space: with an origin
+      // of 0 they are (bi0 + nx) * dx to the last bit, the next patch's xlo
+      const double hi0 = (lo0 - pd.bi0 * pd.dx) + (double)(pd.bi0 + pd.nx) * pd.dx;
+      const double hi1 = (lo1 - pd.bj0 * pd.dy) + (double)(pd.bj0 + pd.ny) * pd.dy;
       for (int k = 0; k < nmics; k++) {
         const double x = mic_x[k], y = mic_y[k];
         if (!(x >= lo0 && x <= hi0 && y >= lo1 && y <= hi1)) continue;

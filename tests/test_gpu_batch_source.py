@@ -82,6 +82,51 @@ def test_microphones_in_one_call(nm):
     d.close()
 
 
+@pytest.mark.parametrize("origin", [(0.0, 0.0), (2.5, 0.75), (-3.0, -0.25), (-0.5, 8.0)])
+def test_microphones_on_a_domain_of_any_origin(origin):
+    """A batch made through the C ABI with its lower corner at `origin`: the
+    entries are those of enl_sample_mics called patch by patch with the same
+    geometry.  dx is a power of two, so every bound is exact."""
+    h, whole = hierarchy(64, 24)
+    lib, desc = whole.lib, np.zeros(len(h.patches), dtype=_lib.PATCH_DESC_DTYPE)
+    for p in h.patches:
+        dx = h.dx(p.level)
+        desc[p.pid] = (p.level, p.box, (origin[0] + p.box[0] * dx, origin[1] + p.box[2] * dx), (dx, dx))
+    handle = ctypes.c_void_p()
+    _lib.check(lib.enl_batch_create(len(desc), desc.ctypes.data_as(ctypes.POINTER(_lib.EnlPatchDesc)), h.g, h.ratio,
+                                    ctypes.byref(handle)))
+    rng = np.random.default_rng(5)
+    nm = 90
+    x, y = origin[0] + rng.uniform(-0.3, 1.3, nm), origin[1] + rng.uniform(-0.3, 1.3, nm)
+    x[::4] = origin[0] + np.round((x[::4] - origin[0]) * 64) / 64  # on cell and patch edges
+    want, P = [], []
+    for p in h.patches:
+        P.append(rng.uniform(1.0, 2.0, size=(p.Ny, p.Nx)))
+        a = ctypes.c_void_p(P[-1].ctypes.data)
+        _lib.check(lib.enl_batch_copy_state(handle, p.pid, 1, None, a, None, None))
+    for lev in range(h.nlevels):
+        dx = h.dx(lev)
+        for p in h.level_patches(lev):
+            lo = desc[p.pid]["xlo"]
+            hi = (lo[0] + p.nx * dx, lo[1] + p.ny * dx)
+            g = p.g
+            v, hit = SRC.sample_mics(p.box, lo, hi, (dx, dx), x, y,
+                                     torch.from_numpy(np.ascontiguousarray(P[p.pid][g:-g, g:-g])).cuda())
+            torch.cuda.synchronize()
+            v, hit = v.cpu().numpy(), hit.cpu().numpy()
+            want += [(k, lev, p.pid, v[k]) for k in np.nonzero(hit)[0]]
+    assert len({m for m, *_ in want}) > nm // 4 and max(m[1] for m in want) == 1
+    room = len(want) + 50
+    mic, level, pid = (np.full(room, -1, np.int32) for _ in range(3))
+    val = np.zeros(room)
+    ptr = lambda a: ctypes.c_void_p(a.ctypes.data)
+    n = lib.enl_batch_sample_mics(handle, nm, ptr(x), ptr(y), room, ptr(mic), ptr(level), ptr(pid), ptr(val))
+    got = [(mic[k], level[k], pid[k], val[k]) for k in range(n)]
+    _lib.check(lib.enl_batch_destroy(handle))
+    whole.close()
+    assert got == want
+
+
 @pytest.mark.parametrize("n0,tile0", [(96, 40), (200, 200)])
 def test_fp32_load_and_store_of_every_patch(n0, tile0):
     """Load carries the FP64 perturbation of the interior, store adds the
