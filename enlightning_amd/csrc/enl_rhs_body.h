@@ -549,15 +549,16 @@ __device__ __forceinline__ void split_compute(const RhsArgs& a, int i0, int j0, 
 
 // LLF speed of a cell in row j (rhs_hybrid_high_llf.m4:270-284): the largest
 // |velocity| + c + c_lr height over the window, along x (dir 0) at the row's
-// height, along y at each point's.  un holds the normal velocity of the
-// points m = -R..R (index m + 3).
+// height, along y at each point's, and never below 0, where the reference's
+// maximum starts.  un holds the normal velocity of the points m = -R..R
+// (index m + 3).
 template <int R>
 __device__ inline double llf_speed(const RhsArgs& a, int j, int dir, const double* un) {
   const double c0 = fma(a.c_lr, fma(a.dy, (double)j + 0.5, a.ylo), a.c), c1 = dir == 0 ? 0.0 : a.c_lr * a.dy;
   double s = fabs(un[3]);
 #pragma unroll
   for (int m = -R; m <= R; m++) s = fmax(s, fma((double)m, c1, fabs(un[m + 3])));
-  return s + c0;
+  return fmax(0.0, s + c0);
 }
 
 // One (direction, component) of a listed WENO cell: the x (dir 0) or y (dir
