@@ -23,7 +23,15 @@ struct PatchDev {
   long src_int;     // interior copy of the source (the drop-in's layout)
   long rhs;         // interior rhs slots, 5*nx*ny
   double dx, dy, xlo, ylo;
+  int chunk0;       // the patch's first chunk (kChunk)
 };
+
+// Passes over every cell of every patch run in chunks of the ghosted boxes, a
+// workgroup and a thread per cell, numbered through all patches: workgroups
+// then follow the cells, whatever the patches' sizes.  (With a grid of the
+// largest patch by the number of patches either one large patch has too few
+// of them or many small ones mostly empty ones.)
+constexpr int kChunk = 256;
 
 // Device copies of one level's fill schedule.
 struct LevelFill {
@@ -55,6 +63,8 @@ struct Batch {
   double* pool = nullptr;
   size_t pool_doubles = 0;
   PatchDev* dp = nullptr;
+  const int* chunk_patch = nullptr;  // the patch of each chunk (device, behind dp)
+  int nchunks = 0;
   int4* tiles = nullptr;
   int ntiles = 0;
   int tile_bx[8], tile_by[8];     // tile shape per level
@@ -129,6 +139,8 @@ inline int upload(Batch* b, T** dst, const T* src, long n) {
   b->allocations.push_back(*dst);
   return check_hip(hipMemcpy(*dst, src, sizeof(T) * (size_t)n, hipMemcpyHostToDevice), "upload batch table");
 }
+
+inline dim3 chunk_grid(const Batch* b) { return dim3((unsigned)b->nchunks); }
 
 // State blocks of RK stage st of an order-stage step: stage 0 reads block 0
 // (the step's start state), stages alternate blocks 1 and 2, the last stage

@@ -853,7 +853,7 @@ int enl_batch_create(int npatch, const enl_patch_desc_t* patches, int gcw, int r
   b->g = gcw;
   b->ratio = ratio;
   b->desc.assign(patches, patches + npatch);
-  long off = 0;
+  long off = 0, chunks = 0;
   for (int p = 0; p < npatch; p++) {
     const enl_patch_desc_t& d = patches[p];
     PatchDev pd;
@@ -887,12 +887,15 @@ int enl_batch_create(int npatch, const enl_patch_desc_t* patches, int gcw, int r
     pd.dy = d.dx[1];
     pd.xlo = d.xlo[0];
     pd.ylo = d.xlo[1];
+    pd.chunk0 = (int)chunks;
+    chunks += (pd.sk + kChunk - 1) / kChunk;
     b->hp.push_back(pd);
     b->cells += (long)pd.nx * pd.ny;
     b->level_cells[d.level] += (long)pd.nx * pd.ny;
     if (d.level + 1 > b->nlevels) b->nlevels = d.level + 1;
   }
   b->pool_doubles = (size_t)off;
+  b->nchunks = (int)chunks;
   hipError_t e = batch_malloc((void**)&b->pool, sizeof(double) * b->pool_doubles);
   if (e != hipSuccess) {
     delete b;
@@ -900,7 +903,16 @@ int enl_batch_create(int npatch, const enl_patch_desc_t* patches, int gcw, int r
   }
   b->allocations.push_back(b->pool);
   (void)hipMemset(b->pool, 0, sizeof(double) * b->pool_doubles);
-  int rc = upload(b, &b->dp, b->hp.data(), npatch);
+  // the patch table and, behind it, the patch of every chunk
+  std::vector<char> table(sizeof(PatchDev) * (size_t)npatch + sizeof(int) * (size_t)chunks);
+  memcpy(table.data(), b->hp.data(), sizeof(PatchDev) * (size_t)npatch);
+  int* of = (int*)(table.data() + sizeof(PatchDev) * (size_t)npatch);
+  for (int p = 0; p < npatch; p++)
+    of = std::fill_n(of, (p + 1 < npatch ? b->hp[p + 1].chunk0 : (int)chunks) - b->hp[p].chunk0, p);
+  char* dev = nullptr;
+  int rc = upload(b, &dev, table.data(), (long)table.size());
+  b->dp = (PatchDev*)dev;
+  b->chunk_patch = (const int*)(dev + sizeof(PatchDev) * (size_t)npatch);
   if (!rc) {
     e = batch_malloc((void**)&b->list, sizeof(unsigned long long) * (size_t)b->cells);
     if (e == hipSuccess) b->allocations.push_back(b->list);

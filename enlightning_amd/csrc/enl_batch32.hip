@@ -718,109 +718,110 @@ __global__ void __launch_bounds__(256) coarsen32_kernel(Fill32 f, double* wc, si
   }
 }
 
-// The conversions below run over every patch in one launch: blockIdx.y walks
-// the patch table, the x blocks a patch's cells.  (One launch per patch, 815
-// of them at the AMR workload, took 4 ms for a store that moves 0.4 GB.)
+// The conversions below run over every patch in one launch, in chunks (kChunk).
+// One launch per patch, 815 of them at the AMR workload, took 4 ms for a store
+// that moves 0.4 GB; one launch of (the largest patch's cells, at most 64
+// workgroups) x patches left a large patch to 64 workgroups.  4096^2 in one
+// patch, load / store: 0.50 / 0.35 ms by the patch, 7.4 / 2.07 ms so, 0.43 /
+// 0.31 ms in chunks; 2048^2 in 1024 patches 6.8 / 7.1, 0.21 / 0.13, 0.13 /
+// 0.13 ms.
 struct Conv32 {
   double* pool;  // FP64 pool
   const PatchDev* pd;
+  const int* chunk_patch;
   const Patch32* p32;
   float* pool32;
   double* wc;
   signed char* res8;
   const double* amb;
-  int npatch;
 };
 
-// The ghosted cell q of a patch: its ambient record, and its interior index
-// (-1 outside the interior).
-__device__ inline const double* conv_cell(const Conv32& c, const Patch32& p, unsigned q, long& ic) {
-  const unsigned row = q / (unsigned)p.sy;
-  const int jj = (int)row - p.g, ii = (int)(q - row * (unsigned)p.sy) - p.g;
-  ic = ii >= 0 && ii < p.nx && jj >= 0 && jj < p.ny ? ii + (long)jj * p.nx : -1;
-  return c.amb + (p.amb + row) * kRec;
-}
+// This thread's cell: its patch, its place in the ghosted box, its ambient
+// record and its interior index (-1 outside the interior).
+struct ConvCell {
+  int y;
+  Patch32 p;
+  long q, ic;
+  const double* rec;
+  bool live;
+  __device__ explicit ConvCell(const Conv32& c) : y(c.chunk_patch[blockIdx.x]), p(c.p32[y]) {
+    const unsigned n = (unsigned)((int)blockIdx.x - c.pd[y].chunk0) * kChunk + threadIdx.x;
+    const unsigned row = n / (unsigned)p.sy;
+    const int jj = (int)row - p.g, ii = (int)(n - row * (unsigned)p.sy) - p.g;
+    live = n < (unsigned)p.sk;
+    q = n;
+    ic = ii >= 0 && ii < p.nx && jj >= 0 && jj < p.ny ? ii + (long)jj * p.nx : -1;
+    rec = c.amb + (p.amb + row) * kRec;
+  }
+};
 
 // FP64 block 0 -> FP32 block 0 (+ carried state, at the patch's offset p.wc
 // of the carried-state pool, and the interior's rounding residuals), and
 // back.
-__global__ void __launch_bounds__(256) to32_kernel(Conv32 c) {
-  for (int y = blockIdx.y; y < c.npatch; y += gridDim.y) {
-    const Patch32& p = c.p32[y];
-    const double* w64 = c.pool + c.pd[y].state[0];
-    float* w32 = c.pool32 + p.blk[0];
-    for (unsigned q = blockIdx.x * 256u + threadIdx.x; q < (unsigned)p.sk; q += gridDim.x * 256u) {
-      long ic;
-      const double* rec = conv_cell(c, p, q, ic);
+__global__ void __launch_bounds__(kChunk) to32_kernel(Conv32 c) {
+  const ConvCell h(c);
+  if (!h.live) return;
+  const Patch32& p = h.p;
+  const double* w64 = c.pool + c.pd[h.y].state[0] + h.q;
+  float* w32 = c.pool32 + p.blk[0] + h.q;
+  double v[7];
 #pragma unroll
-      for (int k = 0; k < 7; k++) {
-        const double v = w64[q + k * p.sk] - amb_of(rec, k);
-        const float vf = (float)v;
-        w32[q + k * p.sk] = vf;
-        if (ic >= 0 && k < 5) {
-          const long o = ic + k * (long)p.nx * p.ny;
-          c.wc[p.wc + o] = v;
-          c.res8[p.res[0] + o] = res_enc(v, vf);
-        }
-      }
+  for (int k = 0; k < 7; k++) v[k] = w64[k * p.sk] - amb_of(h.rec, k);
+  const long nn = (long)p.nx * p.ny;
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    const float vf = (float)v[k];
+    w32[k * p.sk] = vf;
+    if (h.ic >= 0 && k < 5) {
+      c.wc[p.wc + h.ic + k * nn] = v[k];
+      c.res8[p.res[0] + h.ic + k * nn] = res_enc(v[k], vf);
     }
   }
 }
 
-__global__ void __launch_bounds__(256) to64_kernel(Conv32 c) {
-  for (int y = blockIdx.y; y < c.npatch; y += gridDim.y) {
-    const Patch32& p = c.p32[y];
-    double* w64 = c.pool + c.pd[y].state[0];
-    const float* w32 = c.pool32 + p.blk[0];
-    for (unsigned q = blockIdx.x * 256u + threadIdx.x; q < (unsigned)p.sk; q += gridDim.x * 256u) {
-      long ic;
-      const double* rec = conv_cell(c, p, q, ic);
-      double pv[7];
+__global__ void __launch_bounds__(kChunk) to64_kernel(Conv32 c) {
+  const ConvCell h(c);
+  if (!h.live) return;
+  const Patch32& p = h.p;
+  double* w64 = c.pool + c.pd[h.y].state[0] + h.q;
+  const float* w32 = c.pool32 + p.blk[0] + h.q;
+  const double* wc = c.wc + p.wc + h.ic;
+  const long nn = (long)p.nx * p.ny;
+  double pv[7];
 #pragma unroll
-      for (int k = 0; k < 7; k++)
-        pv[k] = ic >= 0 && k < 5 ? c.wc[p.wc + ic + k * (long)p.nx * p.ny] : (double)w32[q + k * p.sk];
+  for (int k = 0; k < 7; k++) pv[k] = h.ic >= 0 && k < 5 ? wc[k * nn] : (double)w32[k * p.sk];
 #pragma unroll
-      for (int k = 0; k < 7; k++) w64[q + k * p.sk] = amb_of(rec, k) + pv[k];
-    }
-  }
+  for (int k = 0; k < 7; k++) w64[k * p.sk] = amb_of(h.rec, k) + pv[k];
 }
 
 // FP64 state block 2 := the ambient on every cell (p, T from the records),
 // FP32 block 2 := 0.
-__global__ void __launch_bounds__(256) ambient_blocks_kernel(Conv32 c) {
-  for (int y = blockIdx.y; y < c.npatch; y += gridDim.y) {
-    const Patch32& p = c.p32[y];
-    double* w64 = c.pool + c.pd[y].state[2];
-    float* w32 = c.pool32 + p.blk[2];
-    for (unsigned q = blockIdx.x * 256u + threadIdx.x; q < (unsigned)p.sk; q += gridDim.x * 256u) {
-      long ic;
-      const double* rec = conv_cell(c, p, q, ic);
+__global__ void __launch_bounds__(kChunk) ambient_blocks_kernel(Conv32 c) {
+  const ConvCell h(c);
+  if (!h.live) return;
+  const Patch32& p = h.p;
+  double* w64 = c.pool + c.pd[h.y].state[2] + h.q;
+  float* w32 = c.pool32 + p.blk[2] + h.q;
 #pragma unroll
-      for (int k = 0; k < 7; k++) {
-        w64[q + k * p.sk] = amb_of(rec, k);
-        w32[q + k * p.sk] = 0.0f;
-      }
-    }
+  for (int k = 0; k < 7; k++) {
+    w64[k * p.sk] = amb_of(h.rec, k);
+    w32[k * p.sk] = 0.0f;
   }
 }
 
 // dK = K64 - K32 on the interior (K64 in the w_n components of FP64 block 1).
-__global__ void __launch_bounds__(256) dk_kernel(Conv32 c) {
-  for (int y = blockIdx.y; y < c.npatch; y += gridDim.y) {
-    const Patch32& p = c.p32[y];
-    const double* k64 = c.pool + c.pd[y].state[1];
-    float* dk = c.pool32 + p.dk;
-    const unsigned nn = (unsigned)p.nx * (unsigned)p.ny;
-    for (unsigned q = blockIdx.x * 256u + threadIdx.x; q < nn; q += gridDim.x * 256u) {
-      const unsigned j = q / (unsigned)p.nx, i = q - j * (unsigned)p.nx;
-      const long g = (long)(i + p.g) + (long)(j + p.g) * p.sy;
+__global__ void __launch_bounds__(kChunk) dk_kernel(Conv32 c) {
+  const ConvCell h(c);
+  if (!h.live || h.ic < 0) return;
+  const Patch32& p = h.p;
+  const double* k64 = c.pool + c.pd[h.y].state[1] + h.q;
+  float* dk = c.pool32 + p.dk + h.ic;
+  const long nn = (long)p.nx * p.ny;
+  double v[5];
 #pragma unroll
-      for (int k = 0; k < 5; k++) {
-        const long o = q + k * (long)nn;
-        dk[o] = (float)(k64[g + k * p.sk] - (double)dk[o]);
-      }
-    }
-  }
+  for (int k = 0; k < 5; k++) v[k] = k64[k * p.sk] - (double)dk[k * nn];
+#pragma unroll
+  for (int k = 0; k < 5; k++) dk[k * nn] = (float)v[k];
 }
 
 }  // namespace
@@ -1125,18 +1126,12 @@ Conv32 conv32(Batch* b) {
   c.wc = F->wc;
   c.res8 = F->res8;
   c.amb = F->amb;
-  c.npatch = b->npatch;
+  c.chunk_patch = b->chunk_patch;
   return c;
-}
-// x blocks for the largest patch (at most 64: larger ones loop), one y per patch
-dim3 conv_grid(Batch* b) {
-  long most = 1;
-  for (const PatchDev& pd : b->hp) most = std::max(most, pd.sk);
-  return dim3(grid_for(most, 256, 64), (unsigned)std::min(b->npatch, 65535));
 }
 
 int load32(Batch* b, hipStream_t s) {
-  hipLaunchKernelGGL(to32_kernel, conv_grid(b), dim3(256), 0, s, conv32(b));
+  hipLaunchKernelGGL(to32_kernel, chunk_grid(b), dim3(kChunk), 0, s, conv32(b));
   return check_hip(hipGetLastError(), "FP32 load");
 }
 
@@ -1338,7 +1333,7 @@ int enl_batch_fp32_prepare(void* handle, int variant, const enl_gas_t* gas, cons
   hipStream_t s = lib_stream();
   // K64 of the ambient: FP64 block 2 := ambient, its rhs into block 1
   // and FP32 block 2 := 0 perturbation
-  hipLaunchKernelGGL(ambient_blocks_kernel, conv_grid(b), dim3(256), 0, s, conv32(b));
+  hipLaunchKernelGGL(ambient_blocks_kernel, chunk_grid(b), dim3(kChunk), 0, s, conv32(b));
   rc = batch_eval_rhs64(b, variant, gas, reflect, 2, 1, s);
   if (rc) return rc;
   // K32 of the ambient: FP32 block 2's ghosts filled, K32 into dk
@@ -1358,7 +1353,7 @@ int enl_batch_fp32_prepare(void* handle, int variant, const enl_gas_t* gas, cons
     rc = stage32<true>(b, F->d_eval, lev, s);
   }
   if (rc) return rc;
-  hipLaunchKernelGGL(dk_kernel, conv_grid(b), dim3(256), 0, s, conv32(b));
+  hipLaunchKernelGGL(dk_kernel, chunk_grid(b), dim3(kChunk), 0, s, conv32(b));
   rc = load32(b, s);
   if (!rc) rc = check_hip(hipStreamSynchronize(s), "enl_batch_fp32_prepare");
   F->ready = rc == 0;
@@ -1405,7 +1400,7 @@ int enl_batch_fp32_load(void* handle) {
 int enl_batch_fp32_store(void* handle) {
   Batch* b = (Batch*)handle;
   if (!b || !b->f32 || !b->f32->ready) return set_error(-2, "FP32 form not prepared");
-  hipLaunchKernelGGL(to64_kernel, conv_grid(b), dim3(256), 0, lib_stream(), conv32(b));
+  hipLaunchKernelGGL(to64_kernel, chunk_grid(b), dim3(kChunk), 0, lib_stream(), conv32(b));
   return check_hip(hipGetLastError(), "enl_batch_fp32_store");
 }
 

@@ -2,6 +2,7 @@
 bit: the source of every patch (enl_batch_add_source), the microphones
 (enl_batch_sample_mics) and the FP32 form's store of patches of every size."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -127,7 +128,7 @@ def test_microphones_on_a_domain_of_any_origin(origin):
     assert got == want
 
 
-@pytest.mark.parametrize("n0,tile0", [(96, 40), (200, 200)])
+@pytest.mark.parametrize("n0,tile0", [(96, 40), (200, 200), (72, 24)])  # (24 + 8)^2: whole chunks of 256
 def test_fp32_load_and_store_of_every_patch(n0, tile0):
     """Load carries the FP64 perturbation of the interior, store adds the
     ambient back: amb + (w - amb) on the interior, amb + float(w - amb) in the
@@ -153,3 +154,34 @@ def test_fp32_load_and_store_of_every_patch(n0, tile0):
             want[g:-g, g:-g] = (A + pert)[g:-g, g:-g]
             assert np.array_equal(v[k], want), (p.pid, k)
     d.close()
+
+
+def host_time(f, reps=10):
+    """Seconds of one of `reps` calls of f in a row, the best of five rows."""
+    f()
+    torch.cuda.synchronize()
+    best = np.inf
+    for _ in range(5):
+        t = time.perf_counter()
+        for _ in range(reps):
+            f()
+        torch.cuda.synchronize()
+        best = min(best, (time.perf_counter() - t) / reps)
+    return best
+
+
+def test_fp32_load_and_store_fill_the_chip_whatever_the_patches():
+    """2048^2 cells in one patch and in 1024 of 64^2: the ghosts of the small
+    ones are a quarter more to move, so the one patch takes no longer than
+    they do; twice their time is allowed.  (With workgroups counted per patch,
+    64 at most, it took seven times as long.)"""
+    took = {}
+    for tile0 in (64, 2048):
+        h = amr.build(2048, 4, 4, 1.0, None, tile0=tile0)
+        d = DeviceHierarchy(h, Gas())
+        rows = np.ones(2048 + 8)
+        d.set_ambient(lambda lev: (-4, 1.2 * rows, 0.1 * rows, 350.0 * rows))
+        d.fp32_prepare()
+        took[len(h.patches)] = host_time(d.fp32_load) + host_time(d.fp32_store)
+        d.close()
+    assert took[1] <= 2 * took[1024], took
