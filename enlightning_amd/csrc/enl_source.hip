@@ -101,22 +101,22 @@ __global__ void __launch_bounds__(256) source_kernel(SourceArgs a) {
                     a.type == kLightning ? *o : 0.0);
 }
 
-// The same for every patch of a hierarchy in one launch (blockIdx.y walks the
-// patch table): one launch per patch, ~700 at a 512^2 base, took 4 ms for a
-// source that costs some 10 us to evaluate.
-__global__ void __launch_bounds__(256) batch_source_kernel(double* pool, const PatchDev* __restrict__ pd, int npatch,
-                                                           SourceArgs a) {
-  for (int y = blockIdx.y; y < npatch; y += gridDim.y) {
-    const PatchDev& p = pd[y];
-    const unsigned n = (unsigned)p.nx * (unsigned)p.ny;
-    double* src = pool + p.src + p.g + p.g * p.sy;
-    for (unsigned q = blockIdx.x * 256u + threadIdx.x; q < n; q += gridDim.x * 256u) {
-      const unsigned j = q / (unsigned)p.nx, i = q - j * (unsigned)p.nx;
-      double* o = src + (long)i + (long)j * p.sy;
-      *o = source_value(a, p.xlo + p.dx * ((double)i + 0.5), p.ylo + p.dy * ((double)j + 0.5),
-                        a.type == kLightning ? *o : 0.0);
-    }
-  }
+// The same for every patch of a hierarchy in one launch, in chunks (kChunk)
+// whose ghosts stand still: one launch per patch, ~700 at a 512^2 base, took
+// 4 ms for a source that costs some 10 us to evaluate; one of (the largest
+// patch's cells, at most 256 workgroups) x patches left a large patch short
+// of waves (a channel of 24 segments on 2048^2 in one patch 0.34 ms by the
+// patch, 0.73 so, 0.35 in chunks; on 1024 patches 36, 0.29 and 0.29 ms).
+__global__ void __launch_bounds__(kChunk) batch_source_kernel(double* pool, const PatchDev* __restrict__ pd,
+                                                              const int* __restrict__ chunk_patch, SourceArgs a) {
+  const PatchDev& p = pd[chunk_patch[blockIdx.x]];
+  const unsigned n = (unsigned)((int)blockIdx.x - p.chunk0) * kChunk + threadIdx.x;
+  const unsigned row = n / (unsigned)p.sy;
+  const int i = (int)(n - row * (unsigned)p.sy) - p.g, j = (int)row - p.g;
+  if (i < 0 || i >= p.nx || j < 0 || j >= p.ny) return;
+  double* o = pool + p.src + n;
+  *o = source_value(a, p.xlo + p.dx * ((double)i + 0.5), p.ylo + p.dy * ((double)j + 0.5),
+                    a.type == kLightning ? *o : 0.0);
 }
 
 // Segments of the channel with the quantities of enlightning.C:2215-2232.
@@ -267,10 +267,7 @@ int enl_batch_add_source(void* handle, const enl_source_t* src, int iteration, i
   if (src->type == kLightning && src->nseg == 0) return 0;
   hipStream_t s = lib_stream();
   if (src->type == kLightning && (rc = upload_segments(src, &a, s))) return rc;
-  long most = 1;
-  for (const PatchDev& pd : b->hp) most = std::max(most, (long)pd.nx * pd.ny);
-  hipLaunchKernelGGL(batch_source_kernel, dim3(grid_for(most, 256, 256), (unsigned)std::min(b->npatch, 65535)),
-                     dim3(256), 0, s, b->pool, b->dp, b->npatch, a);
+  hipLaunchKernelGGL(batch_source_kernel, chunk_grid(b), dim3(kChunk), 0, s, b->pool, b->dp, b->chunk_patch, a);
   hipError_t e = hipGetLastError();
   if (a.seg) {
     hipError_t f = hipFreeAsync((void*)a.seg, s);

@@ -185,3 +185,19 @@ def test_fp32_load_and_store_fill_the_chip_whatever_the_patches():
         took[len(h.patches)] = host_time(d.fp32_load) + host_time(d.fp32_store)
         d.close()
     assert took[1] <= 2 * took[1024], took
+
+
+def test_source_fills_the_chip_whatever_the_patches():
+    """A lightning channel of 48 segments, bound by the exponentials of each
+    cell, over the same cells: 1.75 times the small patches' time is allowed
+    to the one patch.  (With at most 256 workgroups of one wave per SIMD each,
+    it took 2.5 times as long.)"""
+    seg = np.array([[0.1, 0.9, 0.4, 0.5], [0.4, 0.5, 0.35, 0.2], [0.35, 0.2, 0.7, 0.1]] * 16)
+    src = SRC.Source(mode=SRC.PULSE, type=SRC.LIGHTNING, spread=0.02, coords=seg)
+    took = {}
+    for tile0 in (64, 2048):
+        h = amr.build(2048, 4, 4, 1.0, None, tile0=tile0)
+        d = DeviceHierarchy(h, Gas())
+        took[len(h.patches)] = host_time(lambda: d.add_source(src, 0, 0, 1e-4))
+        d.close()
+    assert took[1] <= 1.75 * took[1024], took
