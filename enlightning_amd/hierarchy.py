@@ -416,8 +416,8 @@ class DeviceHierarchy:
             if n <= room:
                 break
             room = n
-        for k in range(n):
-            res[mic[k]].append((int(lev[k]), int(pid[k]), float(val[k])))
+        for k, entry in zip(mic[:n].tolist(), zip(lev[:n].tolist(), pid[:n].tolist(), val[:n].tolist())):
+            res[k].append(entry)
         return res
 
     # ---- regrid -------------------------------------------------------------
