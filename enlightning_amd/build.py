@@ -1,9 +1,11 @@
 """Builds libenlightning_hip.so (gfx950) in-tree with hipcc.
 
 Every HIP source is compiled with:
-  -ffp-contract=off   the reference arithmetic has no FMA contraction; keeping
-                      the exact operation order is what makes the kernels agree
-                      with it to the last bit outside exp/log;
+  -ffp-contract=off   the compiler forms no FMA of its own: what the kernels
+                      share with the reference (sensor, tags, pressure) keeps
+                      its bits, and the other expressions, whose fused
+                      multiply-adds are written out, round alike in every
+                      kernel that uses them;
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed FP32 instructions on this hardware pool.
 The stage kernels' sources also take -mllvm -disable-machine-licm: their

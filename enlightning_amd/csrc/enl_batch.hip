@@ -12,8 +12,8 @@
 // does (fill a level's ghosts, then step its patches, then the next level,
 // whose coarse-to-fine ghosts therefore see the coarse level already
 // advanced by this stage):
-//   * the ghost fill of the level from a precomputed schedule (copy /
-//     linear-refine / physical-BC passes: one launch each; the refine reads
+//   * the ghost fill of the level from a precomputed schedule (copies, linear
+//     refinement and the physical boundary in one launch; the refine reads
 //     coarse cells through the coarse patches' ghosts, refreshed after the
 //     coarse level's stage, i.e. coarse interior data as SAMRAI's
 //     temporary coarse level provides);
@@ -926,9 +926,11 @@ int enl_batch_create(int npatch, const enl_patch_desc_t* patches, int gcw, int r
   for (int lev = 0; lev < kMaxLevels; lev++) {
     // Level 0's split kernel: 32 x 8.  The dense kernel of the refined levels:
     // 16 x 8, whose two planes are four waves; one that waits at the barrier
-    // between the directions holds fewer others up than in the sixteen waves
-    // of 32 x 8 (3,072 refined cells a side of 1024 over 48 patches: a step
-    // 662 -> 614 us; 768: 578 -> 536 us).
+    // between the directions holds fewer others up than in the eight waves
+    // of 32 x 8 (a step of a two-level hierarchy over 1024^2 662 -> 614 us,
+    // over 768^2 578 -> 536 us).  The default does not know the variant: with
+    // rhs_weno_* the dense kernel runs on level 0 too and keeps 32 x 8 there
+    // unless enl_batch_set_level_tiles asks for another shape.
     b->tile_bx[lev] = lev ? 16 : 32;
     b->tile_by[lev] = 8;
   }

@@ -2,9 +2,9 @@
 (enl_device.h eos_p_T, log_mid): density ratios around 1, around the reduction
 points 2^k / sqrt 2, across the range 2^-50 .. 2^50 of the fast path and past
 it, entropies of both signs and zero.  Pressure as the oracle's bit for bit,
-temperature within 4 ulps (1e-15) of an extended-precision evaluation: the
-quotients, the logarithm's and the exponential's roundings, each below an ulp
-of a term of order one, and the exponent's magnitude times its own."""
+temperature T0 exp(x) within 1e-15 (1 + |x|) of an extended-precision
+evaluation: the exponential's rounding, and the roundings of x (its quotients',
+and R/c_v = 0.4 times the logarithm's two ulps), which grow with it."""
 import numpy as np
 import pytest
 

@@ -1,9 +1,8 @@
 """Parity of the HIP kernels (called through the C ABI) with the CPU oracle.
 
 Bar (per field, relative L-infinity against the field's max |value|):
-  rhs            <= 1e-12 (the kernels keep the reference operation order and
-                 IEEE division; only exp() in the N2 relaxation term may round
-                 differently), DRP/WENO switch map bit-exact;
+  rhs            <= 1e-12 (flux differences and source in forms that equal the
+                 reference's but for rounding), DRP/WENO switch map bit-exact;
   runge_kutta    bit-exact;
   update_state   pressure bit-exact, temperature <= 1e-14 (exp/log);
   tag_cells      bit-exact;
