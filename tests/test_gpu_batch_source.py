@@ -2,6 +2,7 @@
 bit: the source of every patch (enl_batch_add_source), the microphones
 (enl_batch_sample_mics) and the FP32 form's store of patches of every size."""
 import ctypes
+import math
 import time
 
 import numpy as np
@@ -62,24 +63,73 @@ def test_bad_sources_are_refused():
     d.close()
 
 
-@pytest.mark.parametrize("nm", [1, 127, 400])
-def test_microphones_in_one_call(nm):
-    h, d = hierarchy()
-    rng = np.random.default_rng(nm)
-    x, y = rng.uniform(-0.1, 1.1, size=(2, nm))
-    x[::3], y[::5] = np.round(x[::3] * 96) / 96, np.round(y[::5] * 96) / 96  # on cell and patch edges
-    got = d.sample_mics(x, y)
-    want = [[] for _ in range(nm)]
+def mic_entries(h, d, x, y):
+    """(microphone, level, patch, value) in the order of the reference's files:
+    per level and patch every microphone within the patch's bounds."""
+    out = []
     P = [v[0] for v in d.gather(0x20, ghosted=False)]
     for lev in range(h.nlevels):
         dx = h.dx(lev)
         for p in h.level_patches(lev):
             lo, hi = (p.box[0] * dx, p.box[2] * dx), ((p.box[1] + 1) * dx, (p.box[3] + 1) * dx)
-            for k in range(nm):
+            for k in range(len(x)):
                 if lo[0] <= x[k] <= hi[0] and lo[1] <= y[k] <= hi[1]:
                     i, j = min(int((x[k] - lo[0]) / dx), p.nx - 1), min(int((y[k] - lo[1]) / dx), p.ny - 1)
-                    want[k].append((lev, p.pid, P[p.pid][j, i]))
-    assert got == want and any(len(m) > 2 for m in want + [[0, 0, 0]])
+                    out.append((k, lev, p.pid, P[p.pid][j, i]))
+    return out
+
+
+def microphones(h, nm):
+    """nm places in and around the domain, some on cell and patch edges; the
+    first on the corner that most patches of both levels share."""
+    rng = np.random.default_rng(nm)
+    x, y = rng.uniform(-0.1, 1.1, size=(2, nm))
+    x[::3], y[::5] = np.round(x[::3] * 96) / 96, np.round(y[::5] * 96) / 96
+    fine = [(a * h.dx(1), b * h.dx(1)) for p in h.level_patches(1) for a in (p.box[0], p.box[1] + 1)
+            for b in (p.box[2], p.box[3] + 1)]
+    x[0], y[0] = max(fine, key=lambda c: sum(
+        p.box[0] * h.dx(p.level) <= c[0] <= (p.box[1] + 1) * h.dx(p.level)
+        and p.box[2] * h.dx(p.level) <= c[1] <= (p.box[3] + 1) * h.dx(p.level) for p in h.patches))
+    return x, y
+
+
+@pytest.mark.parametrize("nm", [1, 127, 400])
+def test_microphones_in_one_call(nm):
+    h, d = hierarchy()
+    x, y = microphones(h, nm)
+    want = [[] for _ in range(nm)]
+    for k, lev, pid, v in mic_entries(h, d, x, y):
+        want[k].append((lev, pid, v))
+    assert len(want[0]) > 2 and {lev for lev, _, _ in want[0]} == {0, 1}
+    assert d.sample_mics(x, y) == want
+    d.close()
+
+
+@pytest.mark.parametrize("room", [0, 1, 129])
+def test_microphones_beyond_the_callers_room(room):
+    """The count of all entries comes back whatever the room, with the first
+    `room` of them and nothing behind; the wrapper calls again with more."""
+    h, d = hierarchy()
+    x, y = microphones(h, 400)
+    want = mic_entries(h, d, x, y)
+    assert len(want) > 129
+    mic, level, pid = (np.full(room + 2, -7, np.int32) for _ in range(3))
+    val = np.full(room + 2, -7.0)
+    ptr = lambda a: ctypes.c_void_p(a.ctypes.data)
+    n = d.lib.enl_batch_sample_mics(d.handle, 400, ptr(x), ptr(y), room, ptr(mic), ptr(level), ptr(pid), ptr(val))
+    assert n == len(want)
+    assert list(zip(mic[:room], level[:room], pid[:room], val[:room])) == want[:room]
+    assert all((a[room:] == -7).all() for a in (mic, level, pid, val))
+    d.close()
+    # the wrapper starts with room for two entries per microphone and level: a
+    # corner on which four patches of each level meet has eight
+    quarters = [(0, 11, 0, 11), (12, 23, 0, 11), (0, 11, 12, 23), (12, 23, 12, 23)]
+    fine = [(32, 47, 32, 47), (48, 63, 32, 47), (32, 47, 48, 63), (48, 63, 48, 63)]
+    h = amr.from_boxes(24, 4, 4, 1.0, [(0, *q) for q in quarters] + [(1, *q) for q in fine])
+    d = DeviceHierarchy(h, Gas())
+    d.load_initial(None, [np.full((5, p.Ny, p.Nx), 1.1 + p.pid) for p in h.patches])
+    got = d.sample_mics([0.5], [0.5])[0]
+    assert len(got) == 8 and [(0, *q) for q in got] == mic_entries(h, d, [0.5], [0.5])
     d.close()
 
 
@@ -140,6 +190,10 @@ def test_fp32_load_and_store_of_every_patch(n0, tile0):
     d.set_ambient(rows)
     d.fp32_prepare()
     before = d.gather(0x7F)
+    # p and T of the ambient, update_state.m4:88-105 as the library's host forms them (c_lr = 0)
+    ambient_p = lambda r, rs: gas.c * gas.c * ((r - gas.rho0) + (gas.gamma1 - 1) / (2 * gas.rho0) * (
+        (r - gas.rho0) * (r - gas.rho0)) + r / gas.c_p * (rs / r)) + gas.p0
+    ambient_T = lambda r, rs: gas.T0 * math.exp((rs / r - gas.R * math.log(gas.rho0 / r)) / gas.c_v)
     d.fp32_load()
     d.fp32_store()
     after = d.gather(0x7F)
@@ -147,11 +201,13 @@ def test_fp32_load_and_store_of_every_patch(n0, tile0):
         _, r, rs, rt = rows(p.level)
         at = slice(p.box[2], p.box[3] + 2 * p.g + 1)
         g = p.g
-        for k, amb in ((0, r), (1, 0 * r), (2, 0 * r), (3, rs), (4, rt)):
+        rp, rT = (np.array([f(*q) for q in zip(r.tolist(), rs.tolist())]) for f in (ambient_p, ambient_T))
+        for k, amb in ((0, r), (1, 0 * r), (2, 0 * r), (3, rs), (4, rt), (5, rp), (6, rT)):
             A = amb[at][:, None]
             pert = u[k] - A
             want = A + pert.astype(np.float32).astype(np.float64)
-            want[g:-g, g:-g] = (A + pert)[g:-g, g:-g]
+            if k < 5:
+                want[g:-g, g:-g] = (A + pert)[g:-g, g:-g]
             assert np.array_equal(v[k], want), (p.pid, k)
     d.close()
 

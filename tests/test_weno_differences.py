@@ -10,10 +10,43 @@ reference's own.  Stratified, smooth, shocked, constant and random stencils.
 import numpy as np
 import pytest
 
-from tests.test_weno_combination import EPS, C1_6, C13_12, W01, W03, W06, L, divergence, reference
-
+L = np.longdouble
 pytestmark = pytest.mark.skipif(np.finfo(L).eps >= np.finfo(np.float64).eps, reason="needs extended long double")
+C13_12, EPS, C1_6 = (L(np.float32(v)) for v in (13.0 / 12.0, 10.0e-6, 1.0 / 6.0))
+W01, W06, W03 = (L(np.float32(v)) for v in (0.1, 0.6, 0.3))
 C1_3, C2_3 = (L(np.float32(a) / np.float32(3)) for a in (1.0, 2.0))
+
+
+def parts(a, b, c, d, e, T, plus):
+    b0 = T(C13_12) * (c - 2 * d + e) ** 2 + T(0.25) * (3 * c - 4 * d + e) ** 2
+    b1 = T(C13_12) * (b - 2 * c + d) ** 2 + T(0.25) * (b - d) ** 2
+    b2 = T(C13_12) * (a - 2 * b + c) ** 2 + T(0.25) * (a - 4 * b + 3 * c) ** 2
+    if plus:  # wenop
+        cs = (T(W03), T(W06), T(W01))
+        f = (T(C1_6) * (2 * c + 5 * d - e), T(C1_6) * (-b + 5 * c + 2 * d), T(C1_6) * (2 * a - 7 * b + 11 * c))
+    else:  # wenom
+        cs = (T(W01), T(W06), T(W03))
+        f = (T(C1_6) * (11 * c - 7 * d + 2 * e), T(C1_6) * (2 * b + 5 * c - d), T(C1_6) * (-a + 5 * b + 2 * c))
+    D = [(T(EPS) + x) ** 2 for x in (b0, b1, b2)]
+    return cs, D, f
+
+
+def reference(cs, D, f):
+    z = [c / d for c, d in zip(cs, D)]
+    s = z[0] + z[1] + z[2]
+    return (z[0] / s) * f[0] + (z[1] / s) * f[1] + (z[2] / s) * f[2]
+
+
+def divergence(form, T, fp, fm):
+    """p1 + m1 - p2 - m2 at every cell (rhs_hybrid_high_llf.m4:286-354)."""
+    out = []
+    for i in range(3, len(fp) - 3):
+        p1 = form(*parts(*fp[i - 3:i + 2], T, True))
+        m1 = form(*parts(*fm[i - 2:i + 3], T, False))
+        p2 = form(*parts(*fp[i - 2:i + 3], T, True))
+        m2 = form(*parts(*fm[i - 1:i + 4], T, False))
+        out.append(p1 + m1 - p2 - m2)
+    return np.array(out)
 
 
 def pair5(e, T):
