@@ -129,8 +129,8 @@ __device__ inline double rcp_cubic(double d) {
 // and alpha w (the pressure, a stratified ambient) cancels in the first
 // subtraction, before anything is rounded at its size.  Where the products
 // leave the finite range (16 beta beyond ~1e38, or non-finite data) the
-// result is not finite and the caller evaluates the reference's weights
-// instead (REF, weno_pair5_ref).  A pass of one all-WENO RK3 step at 1024^2:
+// result is not finite and the caller evaluates the reference's expressions
+// instead (weno_dir_ref).  A pass of one all-WENO RK3 step at 1024^2:
 // 398 us with four separate reconstructions of one division each, 291 us in
 // this form, 307 us with the candidates taken relative to their middle point
 // instead of f_1 (three more operations per sign, no smaller error on any
@@ -140,18 +140,16 @@ __device__ inline double rcp_cubic(double d) {
 constexpr double kR2 = kW01 / kW06;
 static_assert(kW03 / kW06 == 0.5, "the float literals 0.3 and 0.6 differ by an exact factor of two");
 
-__device__ inline double weno_pair5_ref(double e0, double e1, double e2, double e3, double e4) {
-  const double c1 = e1 - e0, c2 = e2 - e1, c3 = e3 - e2, c4 = e4 - e3;
-  auto one = [](double d0, double l0, double d1, double l1, double d2, double l2) {
-    const double b0 = 0.25 * (kC13_12 * sq(d0) + 0.25 * sq(l0));
-    const double b1 = 0.25 * (kC13_12 * sq(d1) + 0.25 * sq(l1));
-    const double b2 = 0.25 * (kC13_12 * sq(d2) + 0.25 * sq(l2));
-    const double z0 = kW03 / sq(kEpsWeno + b0), z1 = kW06 / sq(kEpsWeno + b1), z2 = kW01 / sq(kEpsWeno + b2);
-    const double sigma = z0 + z1 + z2;
-    return (z0 / sigma) * (d0 - d1) + 2 * ((z2 / sigma) * (d1 - d2));
-  };
-  return (e1 - 5 * e2 - 2 * e3) - one(c3, e3 - 3 * e2, c2, e1 + e2, c1, 3 * e1 - e0) +
-         one(c4, e4 - 3 * e3, c3, e2 + e3, c2, 3 * e2 - e1);
+// The reference's reconstruction wenop5 (rhs_hybrid_high_llf.m4:400-433) by its
+// own expressions; wenom5 (365-398) is its mirror image, (e, d, c, b, a).
+__device__ inline double wenop5_ref(double a, double b, double c, double d, double e) {
+  const double b0 = kC13_12 * sq(c - 2 * d + e) + 0.25 * sq(3 * c - 4 * d + e);
+  const double b1 = kC13_12 * sq(b - 2 * c + d) + 0.25 * sq(b - d);
+  const double b2 = kC13_12 * sq(a - 2 * b + c) + 0.25 * sq(a - 4 * b + 3 * c);
+  const double z0 = kW03 / sq(kEpsWeno + b0), z1 = kW06 / sq(kEpsWeno + b1), z2 = kW01 / sq(kEpsWeno + b2);
+  const double sigma = z0 + z1 + z2;
+  return (z0 / sigma) * (kC1_6 * (2 * c + 5 * d - e)) + (z1 / sigma) * (kC1_6 * (-b + 5 * c + 2 * d)) +
+         (z2 / sigma) * (kC1_6 * (2 * a - 7 * b + 11 * c));
 }
 
 __device__ inline double weno_pair5(double e0, double e1, double e2, double e3, double e4) {
@@ -184,13 +182,11 @@ __device__ inline double weno_pair5(double e0, double e1, double e2, double e3, 
 // operations and its error on random data is 1.4 times the reference's.
 static_assert(kC2_3 == 2 * kC1_3, "float(2/3) = 2 float(1/3)");
 
-__device__ inline double weno_pair3_ref(double e1, double e2, double e3) {
-  auto one = [](double a, double b) {
-    const double z0 = kC2_3 / sq(kEpsWeno + 0.25 * sq(b)), z1 = kC1_3 / sq(kEpsWeno + 0.25 * sq(a));
-    const double sigma = z0 + z1;
-    return (z0 / sigma) * b + (z1 / sigma) * a;
-  };
-  return one(e1, e2) - one(e2, e3) - 2 * e2;
+// wenop3 (rhs_hybrid_low_llf.m4:375-399); wenom3 (349-373) is its mirror image.
+__device__ inline double wenop3_ref(double a, double b, double c) {
+  const double z0 = kC2_3 / sq(kEpsWeno + sq(c - b)), z1 = kC1_3 / sq(kEpsWeno + sq(b - a));
+  const double sigma = z0 + z1;
+  return (z0 / sigma) * (0.5 * (b + c)) + (z1 / sigma) * (0.5 * (-a + 3 * b));
 }
 __device__ inline double weno_pair3(double e1, double e2, double e3) {
   constexpr double kE = 4 * kEpsWeno;
@@ -207,7 +203,7 @@ __device__ inline double weno_pair3(double e1, double e2, double e3) {
 template <int ORDER>
 constexpr double kWenoUnit = ORDER == 5 ? 0.5 * kC1_6 : 0.25;
 
-template <int ORDER, bool REF>
+template <int ORDER>
 __device__ inline double weno_dir(const double* F, const double* W, double alpha) {
   constexpr int R = ORDER == 5 ? 3 : 2;
   double dF[6], dW[6];
@@ -218,17 +214,47 @@ __device__ inline double weno_dir(const double* F, const double* W, double alpha
   }
   auto ep = [&](int m) { return fma(alpha, dW[m], dF[m]); };
   auto em = [&](int m) { return fma(-alpha, dW[m], dF[m]); };
-  if constexpr (ORDER == 5 && REF)
-    return weno_pair5_ref(ep(0), ep(1), ep(2), ep(3), ep(4)) + weno_pair5_ref(em(5), em(4), em(3), em(2), em(1));
-  else if constexpr (ORDER == 5) {
+  if constexpr (ORDER == 5) {
     const double p = weno_pair5(ep(0), ep(1), ep(2), ep(3), ep(4));
     __builtin_amdgcn_sched_barrier(0);
     return p + weno_pair5(em(5), em(4), em(3), em(2), em(1));
-  }
-  else if constexpr (REF)
-    return weno_pair3_ref(ep(1), ep(2), ep(3)) + weno_pair3_ref(em(4), em(3), em(2));
-  else
+  } else
     return weno_pair3(ep(1), ep(2), ep(3)) + weno_pair3(em(4), em(3), em(2));
+}
+
+// The same by the reference's expressions, for where weno_dir's is not finite:
+// its weights vanish for a candidate across a jump whose smoothness leaves the
+// range, and the other candidates are summed as they are (the differences of
+// weno_dir would hold the jump and lose them in it).  point(m, F, W) gives F
+// and W at point m.  pf1, mf1, pf2 and mf2 come from one rolled loop that reads
+// its points again: rare, and no registers of the path before it are held for
+// it (dense kernel 81 VGPRs, 114 with the four written out; the list kernel 154
+// and no spills, 168 and 36 B with the stencil selected into registers:
+// channel at 2048^2 2.70 -> 2.63 ms).
+template <int ORDER, class Point>
+__device__ inline double weno_dir_ref(Point point, double alpha) {
+  constexpr int R = ORDER == 5 ? 3 : 2;
+  double sum = 0;
+#pragma unroll 1
+  for (int r = 0; r < 4; r++) {
+    const bool minus = r & 1, second = r >> 1;
+    const int first = (minus ? R - 1 : -R) + second, step = minus ? -1 : 1;
+    const double s = minus ? -alpha : alpha;
+    double f[2 * R - 1];
+#pragma unroll
+    for (int q = 0; q < 2 * R - 1; q++) {
+      double F, W;
+      point(first + q * step, F, W);
+      f[q] = 0.5 * (F + s * W);
+    }
+    double v;
+    if constexpr (ORDER == 5)
+      v = wenop5_ref(f[0], f[1], f[2], f[3], f[4]);
+    else
+      v = wenop3_ref(f[0], f[1], f[2]);
+    sum = r == 0 ? v : second ? sum - v : sum + v;
+  }
+  return sum / kWenoUnit<ORDER>;
 }
 
 // Smoothness ratio of the hybrid sensor and of tag_cells

@@ -3,7 +3,6 @@
 // hierarchy kernels (enl_batch.hip).  See enl_rhs.hip for the design.
 #pragma once
 #include <cmath>
-#include <type_traits>
 
 #include "enl_device.h"
 #include "enl_kernels.h"
@@ -608,13 +607,12 @@ __device__ __forceinline__ double list_item(const RhsArgs& a, int cell, int dir,
   }
 #pragma unroll
   for (int m = -R; m <= R; m++) F[m + 3] = fma(W[m + 3], un[m + 3], pr[m + 3]);
-  double d = weno_dir<Sc::order, false>(F, W, alpha);
+  double d = weno_dir<Sc::order>(F, W, alpha);
   if (!__builtin_isfinite(d)) {
-    // by the reference's weights; the stencil is formed again, not kept for this
+    // by the reference's expressions; the stencil is formed again, not kept for this
     long at = g;
     asm volatile("" : "+v"(at) : : "memory");
-#pragma unroll 1
-    for (int m = -R; m <= R; m++) {
+    auto point = [&](int m, double& f, double& x) {
       const long q = at + m * step;
       const double w0 = a.w[q];
       double p = 0, T;
@@ -624,15 +622,10 @@ __device__ __forceinline__ double list_item(const RhsArgs& a, int cell, int dir,
         else
           p = a.p[q];
       }
-      const double x = a.w[q + k * G.sk], f = fma(x, a.w[q + kn] * rcp_any(w0), p);
-#pragma unroll
-      for (int n = 0; n < 7; n++)
-        if (n == m + 3) {
-          W[n] = x;
-          F[n] = f;
-        }
-    }
-    d = weno_dir<Sc::order, true>(F, W, alpha);
+      x = a.w[q + k * G.sk];
+      f = fma(x, a.w[q + kn] * rcp_any(w0), p);
+    };
+    d = weno_dir_ref<Sc::order>(point, alpha);
   }
   return d * (dir == 0 ? a.weno_x : a.weno_y);
 }
@@ -743,7 +736,7 @@ __device__ __forceinline__ void list_block(ArgsOf args_of, const unsigned long l
 // each component keeps the next one's loads out of its live range (104 VGPRs
 // against 127 at 1024^2 all-WENO: 291 against 300 us per step).  Components
 // whose WENO products left the finite range are evaluated again by the
-// reference's weights in a rolled loop behind them.  The x plane's results
+// reference's expressions (weno_dir_ref) in a rolled loop behind them.  The x plane's results
 // meet the y plane's in LDS (xs: X then H, 10 x BX*BY doubles) and the y
 // plane forms each component as (X + Y) + H,
 // the reference's order, and writes the cell.  One direction per thread
@@ -810,19 +803,26 @@ __device__ __forceinline__ void dense2_body(const RhsArgs& a, int i0, int j0, De
 #pragma unroll
     for (int m = -R; m <= R; m++) un[m + 3] = L.u[e + m];
     const double af = Sc::llf ? llf_speed<R>(a, j, 0, un) : a.alpha;
-    auto term = [&](int k, auto ref) {
+    auto term = [&](int k) {
       double F[7], W[7];
 #pragma unroll
       for (int m = -R; m <= R; m++) {
         W[m + 3] = L.w[k][e + m];
         F[m + 3] = fma(W[m + 3], un[m + 3], k == 1 ? L.p[e + m] : 0.0);
       }
-      return weno_dir<Sc::order, decltype(ref)::value>(F, W, af) * a.weno_x;
+      return weno_dir<Sc::order>(F, W, af) * a.weno_x;
+    };
+    auto again = [&](int k) {
+      auto point = [&](int m, double& f, double& w) {
+        w = L.w[k][e + m];
+        f = fma(w, L.u[e + m], k == 1 ? L.p[e + m] : 0.0);
+      };
+      return weno_dir_ref<Sc::order>(point, af) * a.weno_x;
     };
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < 5; k++) {
-      const double x = term(k, std::false_type());
+      const double x = term(k);
       xs[k * Sh::threads + c] = x;
       bad = bad || !__builtin_isfinite(x);
       __builtin_amdgcn_sched_barrier(0);
@@ -830,33 +830,40 @@ __device__ __forceinline__ void dense2_body(const RhsArgs& a, int i0, int j0, De
     if (bad) {
 #pragma unroll 1
       for (int k = 0; k < 5; k++)
-        if (!__builtin_isfinite(xs[k * Sh::threads + c])) xs[k * Sh::threads + c] = term(k, std::true_type());
+        if (!__builtin_isfinite(xs[k * Sh::threads + c])) xs[k * Sh::threads + c] = again(k);
     }
   } else if (live) {
     double un[7];
 #pragma unroll
     for (int m = -R; m <= R; m++) un[m + 3] = L.v[e + m * S];
     const double ag = Sc::llf ? llf_speed<R>(a, j, 1, un) : a.alpha;
-    auto term = [&](int k, auto ref) {
+    auto term = [&](int k) {
       double F[7], W[7];
 #pragma unroll
       for (int m = -R; m <= R; m++) {
         W[m + 3] = L.w[k][e + m * S];
         F[m + 3] = fma(W[m + 3], un[m + 3], k == 2 ? L.p[e + m * S] : 0.0);
       }
-      return weno_dir<Sc::order, decltype(ref)::value>(F, W, ag) * a.weno_y;
+      return weno_dir<Sc::order>(F, W, ag) * a.weno_y;
+    };
+    auto again = [&](int k) {
+      auto point = [&](int m, double& f, double& w) {
+        w = L.w[k][e + m * S];
+        f = fma(w, L.v[e + m * S], k == 2 ? L.p[e + m * S] : 0.0);
+      };
+      return weno_dir_ref<Sc::order>(point, ag) * a.weno_y;
     };
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < 5; k++) {
-      Y[k] = term(k, std::false_type());
+      Y[k] = term(k);
       bad = bad || !__builtin_isfinite(Y[k]);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (bad) {
 #pragma unroll 1
       for (int k = 0; k < 5; k++) {
-        const double y = term(k, std::true_type());
+        const double y = again(k);
 #pragma unroll
         for (int q = 0; q < 5; q++)
           if (q == k && !__builtin_isfinite(Y[q])) Y[q] = y;
