@@ -930,7 +930,8 @@ int enl_batch_create(int npatch, const enl_patch_desc_t* patches, int gcw, int r
     // of 32 x 8 (a step of a two-level hierarchy over 1024^2 662 -> 614 us,
     // over 768^2 578 -> 536 us).  The default does not know the variant: with
     // rhs_weno_* the dense kernel runs on level 0 too and keeps 32 x 8 there
-    // unless enl_batch_set_level_tiles asks for another shape.
+    // unless enl_batch_set_level_tiles asks for another shape (1024^2 in 64^2
+    // patches: 298 us a step, with 16 x 8 278).
     b->tile_bx[lev] = lev ? 16 : 32;
     b->tile_by[lev] = 8;
   }

@@ -297,8 +297,9 @@ int enl_batch_prepare(void *handle, const int *reflect);
 int enl_batch_add_source(void *handle, const enl_source_t *src, int iteration, int pulse_time0, double dt);
 /* The microphones' pressure read (enl_sample_mics) over the hierarchy: for
  * every level in order, every patch of it in pid order and every microphone
- * within the patch's bounds (inclusive), one entry: the microphone's index,
- * level, pid and the pressure of its cell.  All arrays are host memory.
+ * within the patch's bounds (inclusive; xlo, and the origin xlo - box[0] dx
+ * plus (box[1] + 1) dx), one entry: the microphone's index, level, pid and the
+ * pressure of its cell.  All arrays are host memory.
  * Writes at most max_entries entries and returns how many there are (call
  * again with more room when that is larger), or a negative error code. */
 int enl_batch_sample_mics(void *handle, int nmics, const double *mic_x, const double *mic_y, int max_entries, int *mic,
