@@ -13,8 +13,12 @@ from enlightning_amd import _lib, amr
 from enlightning_amd import source as SRC
 from enlightning_amd.gas import Gas
 from enlightning_amd.hierarchy import DeviceHierarchy
+from tests import devops as D
 
 pytestmark = pytest.mark.gpu
+
+if D.DRY:
+    pytest.skip("the one-launch forms have no CPU stand-in", allow_module_level=True)
 
 
 def hierarchy(n0=96, tile0=40):
